@@ -327,15 +327,19 @@ __device__ __forceinline__ void jacobi_load(double* a, double* v, const T* A, in
 }
 
 // Descending order of the diagonal of a: thread i places index i at its rank (ties by
-// index), so order is a permutation.
+// index, NaN as +Inf), so order is a permutation for every matrix: its entries address LDS.
 template <int LD = SJLD>
 __device__ __forceinline__ void jacobi_order(const double* a, int np, int* order) {
   const int i = threadIdx.x;
   if (i < np) {
-    const double di = a[i * LD + i];
+    auto key = [&](int j) {
+      const double d = a[j * LD + j];
+      return d == d ? d : (double)INFINITY;
+    };
+    const double di = key(i);
     int rank = 0;
     for (int j = 0; j < np; ++j) {
-      const double dj = a[j * LD + j];
+      const double dj = key(j);
       rank += (dj > di || (dj == di && j < i)) ? 1 : 0;
     }
     order[rank] = i;
