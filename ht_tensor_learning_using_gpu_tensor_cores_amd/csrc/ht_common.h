@@ -13,6 +13,13 @@ namespace ht {
 
 int hip_fail(hipError_t e, const char* what);
 
+// Householder QR: a column whose remaining squared norm is at most this is taken as zero (no
+// reflector). Each exactly dependent column is ~1e-16 of the one before, so squares reach the
+// subnormal numbers after some nine of them; their few digits give a tau that does not fit its
+// vector, and the product of such reflectors is far from orthogonal (up to Inf after 20
+// columns). FP32 input starts at 1e-45, rounding of it at 1e-61.
+constexpr double HH_TINY = 1e-290;
+
 // ---------------------------------------------------------------- MFMA operand types
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));

@@ -37,7 +37,7 @@ __device__ void block_householder(double* A, double* tau, double* red, double* n
       double sub = 0.0;
       for (int g = 0; g < ng; ++g) sub += nrm[g];
       const double alpha = A[j * ld + j];
-      if (sub == 0.0) {
+      if (sub <= HH_TINY) {
         sh_tau = 0.0; sh_beta = alpha; sh_scale = 0.0;
       } else {
         const double nr = sqrt(alpha * alpha + sub);

@@ -923,7 +923,7 @@ __global__ __launch_bounds__(1024) void qr_kernel(const double* __restrict__ Y, 
       for (int w = 0; w < SW; ++w) sub += nrm[w];
       const double alpha = alpha_s;
       double tau = 0.0, scale = 0.0, beta = alpha;
-      if (sub > 0.0) {
+      if (sub > HH_TINY) {
         const double nr = sqrt(alpha * alpha + sub);
         beta = alpha >= 0.0 ? -nr : nr;
         tau = (beta - alpha) / beta;
