@@ -35,9 +35,11 @@ def test_tsqr_deficient(lib, handle, m, b):
         np.testing.assert_allclose(q @ r64, Y, atol=1e-5, err_msg=str(seed))
 
 
-# 65 to 256 rows: powers of the block, Householder QR, Rayleigh-Ritz. Tolerances of the top-k
-# tests: the values to 1e-10 of the largest (the solver's own), orthonormal to 1e-10.
-@pytest.mark.parametrize("n,k", [(65, 16), (100, 32), (200, 24), (256, 32)])
+# 65 to 256 rows: powers of the block, Householder QR, Rayleigh-Ritz; 64 rows, more than 32
+# pairs: Jacobi of the matrix. Blocks of 48 columns and more leave Jacobi entries down to the
+# subnormal numbers. Tolerances of the top-k tests: values to 1e-10 of the largest (the solver's
+# own), orthonormal to 1e-10.
+@pytest.mark.parametrize("n,k", [(64, 40), (65, 16), (96, 64), (100, 32), (127, 63), (128, 64), (200, 24), (256, 32)])
 def test_topk_deficient(lib, handle, n, k):
     import torch
     for seed in range(24):
