@@ -830,9 +830,10 @@ int Engine::view_gemm(const float* x, PMS v, int op, const float* B, int b, int 
 // The blocks are orthonormalised by shifted CholeskyQR (an intermediate left block, which
 // only carries the span into the next product, by its first pass alone), and the Ritz values
 // of an iteration are the eigenvalues of Y^T Y, Y = A Qz. A non-positive pivot (an exactly
-// rank-deficient block) repeats the iteration with TSQR. On 64^4 at rank 16 (4096 x 4096,
-// blocks of 32) an iteration's two TSQRs, chains of ~220 us levels, took 1.7 ms; four CholeskyQR
-// passes of ~40 us (15 us of them the b x b factor), with products and eigenvalues, 0.3 ms.
+// rank-deficient block: a constant tensor, a few entries, zeros outside a box) or a value that
+// is not finite repeats the iteration with TSQR. On 64^4 at rank 16 (4096 x 4096, blocks of 32)
+// an iteration's two TSQRs, chains of ~220 us levels, took 1.7 ms; four CholeskyQR passes of
+// ~40 us (15 us of them the b x b factor), with products and eigenvalues, 0.3 ms.
 int Engine::exact_svd_subspace(const float* x, PMS v, int kU, int kW, double* U, double* Wr, double* sv,
                                uint32_t stream) {
   const auto mk = arena->mark();
@@ -913,11 +914,13 @@ int Engine::svd_subspace(const float* x, PMS v, int kU, int kW, double* U, doubl
     int bad = 0;
     std::memcpy(cur.data(), host.data(), sizeof(double) * b);
     std::memcpy(&bad, host.data() + sizeof(double) * b, sizeof(int));
-    if (!std::isfinite(cur[0])) return HT_ERR_NONFINITE;
-    if (bad) {
+    // A failed pivot left an arbitrary basis, and the Gaussian block's products are ~sqrt(rows)
+    // larger than an orthonormal one's: what is not finite here may be with TSQR.
+    if (!by_tsqr && (bad || !std::isfinite(cur[0]))) {
       *deficient = 1;
       return 0;
     }
+    if (!std::isfinite(cur[0])) return HT_ERR_NONFINITE;
     double diff = 0.0;
     for (int i = 0; i < kk; ++i) {
       diff = std::max(diff, std::fabs(cur[i] - prev[i]));

@@ -417,12 +417,11 @@ __global__ __launch_bounds__(KP <= 32 ? 64 : 128) __attribute__((amdgpu_waves_pe
     double* c = &col[k & 1][1 - (k & 1)];  // entry k + 1 of it is 16-byte aligned
     double ri = 0.0;
     if (ONE || part == 0) {
-      double d = lane_bcast(r[0], k);
-      if (!(d > 0.0)) {
-        bad = 1;
-        d = 1e-300;
-      }
-      ri = rsq_nr(d);
+      // a pivot that is not positive sets info and drops its column (l = 0), so that the
+      // later steps, and what is formed of the flagged factor, stay finite
+      const double d = lane_bcast(r[0], k);
+      if (d > 0.0) ri = rsq_nr(d);
+      else bad = 1;
     }
     if constexpr (!ONE) {
       if (part == 0) {
