@@ -426,7 +426,7 @@ __global__ __launch_bounds__(1024) void power_reg_kernel(const TG* __restrict__ 
       tr += part[1][w];
     }
     __syncthreads();
-    const bool decays = tr * tr < (double)b * f2;
+    const bool decays = tr * tr < (double)kdec * f2;
     if (c0 == 0 && tid == 0 && beff) {
       beff[bidx] = decays ? kdec : b;
       beff[gridDim.y + bidx] = decays;
@@ -1236,14 +1236,16 @@ int topk_small_launch(hipStream_t st, const double* A, long sA, int n, int k, do
 }
 
 // kdec > 0 (mode 0 from a generated block, k = kdec wanted columns): the q powers are meant
-// for a flat spectrum. One whose effective rank tr(G)^2 / ||G||_F^2 is below the block's width
-// b decays within the block; q = 24 powers would collapse the wanted directions onto the top
-// one (theta_k / theta_1 = 0.16: 0.16^24 = 8e-20), and columns past the rank would become
-// rounding noise. Such a problem takes two powers, its columns past k stay random for the
-// next round, should there be one, and beff[problem] = k tells qr_kernel and rr_kernel to work
-// on k columns (b otherwise); beff[batch + problem] is the outcome of the test. 256 rows of
-// rank 16, b = 32: one round of 127 us in the place of two, the first with a Householder QR,
-// of 510.
+// for a flat spectrum. One whose effective rank tr(G)^2 / ||G||_F^2 is below k decays within
+// the wanted columns; q = 24 powers would collapse them onto the top one (theta_k / theta_1 =
+// 0.16: 0.16^24 = 8e-20), and columns past the rank would become rounding noise. Such a problem
+// takes two powers, its columns past k stay random for the next round, should there be one, and
+// beff[problem] = k tells qr_kernel and rr_kernel to work on k columns (b otherwise);
+// beff[batch + problem] is the outcome of the test. 256 rows of rank 16, b = 32: one round of
+// 127 us in the place of two, the first with a Householder QR, of 510. Between k and b the 24
+// powers of the whole block are right: they end a spectrum of 25 values at 16 pairs in one
+// round, where two powers of k columns miss twice (a 32^4 call 0.70 against 1.05 ms); a spectrum
+// without an end (i^-1/2, k = 6) loses by them (1.17 against 1.05 ms).
 // G32, when given, is an FP32 copy of G that modes 0 and 2 read instead; mode 1 always
 // reads G. Filter steps keep G in registers (power_reg_kernel, one column per work-group)
 // for FP32 G and for FP64 G with n <= 128; the rest take power_kernel, two columns per
