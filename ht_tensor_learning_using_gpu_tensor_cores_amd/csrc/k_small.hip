@@ -118,8 +118,10 @@ __device__ __forceinline__ void topk_jacobi(double* a, double* v, int* order, co
 
 // The k largest eigenpairs (k <= 32) of symmetric n x n matrices, n <= 64, one work-group
 // each: U (n x k) with canonical signs and w (k), descending, by tridiagonalisation (k_tri.h);
-// a problem whose result fails that method's checks (clustered wanted eigenvalues, a zero or
-// non-finite matrix) takes the full Jacobi. NR registers per lane hold a row. n <= 32: 512
+// a problem whose result fails that method's checks (equal wanted eigenvalues, a non-finite
+// matrix) takes the full Jacobi. A diagonal matrix (the Grams of an identity, zero) is only
+// sorted: its equal eigenvalues would run the method in vain (64^4 identity by leaves-to-root,
+// a call: 809 -> 603 us, 691 with Jacobi). NR registers per lane hold a row. n <= 32: 512
 // threads, 128 registers are not enough but 256 are, and Jacobi can follow in the same
 // kernel. n <= 64 needs 256 threads for its registers, with which Jacobi would be slower than
 // with 1024: topk_redo_kernel follows (5 us). Against the full Jacobi for every problem,
@@ -140,9 +142,20 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT / 256, NT
   A += bidx * sA;
   U += bidx * sU;
   w += bidx * sw;
+  int off = 0;
 #pragma unroll 8
-  for (int e = tid; e < n * n; e += NT) a[(e % n) * SJLD + e / n] = A[e];
-  __syncthreads();
+  for (int e = tid; e < n * n; e += NT) {
+    const double x = A[e];
+    a[(e % n) * SJLD + e / n] = x;
+    off |= e % n != e / n && x != 0.0;
+  }
+  if (!__syncthreads_or(off)) {  // (also NaN on the diagonal)
+    jacobi_order(a, n, order);
+    __syncthreads();
+    for (int e = tid; e < n * k; e += NT) U[e] = e % n == order[e / n] ? 1.0 : 0.0;
+    if (tid < k) w[tid] = a[order[tid] * SJLD + order[tid]];
+    return;
+  }
   if (wv == 0) {
     const int ok = tri_reduce_wave<SJLD, NR>(a, n, &tri);
     if (lane == 0) ok_s = ok;
