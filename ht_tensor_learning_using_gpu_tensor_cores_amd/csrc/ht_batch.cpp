@@ -101,7 +101,6 @@ ht_status ht_decompose_batched(ht_handle_t h, const float* x, int32_t count, con
   int64_t total = 0;
   int s = describe(count, dims, ranks, &items, &total, nullptr);
   if (s) return (ht_status)s;
-  int nmax = 1;
   std::vector<double> work(count);
   long gsize = 0, bsize = 0;
   int nrows[BT_NMAX + 1] = {};  // eigen problems by number of rows
@@ -111,7 +110,6 @@ ht_status ht_decompose_batched(ht_handle_t h, const float* x, int32_t count, con
     it.out_off = out_offsets[b];
     const double n1 = it.n[0], n2 = it.n[1], n3 = it.n[2];
     work[b] = n1 * n2 * n3 * (n1 + n2 + n3);
-    nmax = std::max(nmax, std::max(it.n[0], std::max(it.n[1], it.n[2])));
     it.g_off = gsize;
     it.u_scr = bsize;
     for (int m = 0; m < 3; ++m) {
@@ -152,33 +150,10 @@ ht_status ht_decompose_batched(ht_handle_t h, const float* x, int32_t count, con
   if (hipMemcpyAsync(itd, items.data(), sizeof(BatchItem) * count, hipMemcpyHostToDevice, h->stream) != hipSuccess ||
       hipMemcpyAsync(ord, order.data(), sizeof(int) * order.size(), hipMemcpyHostToDevice, h->stream) != hipSuccess)
     return HT_ERR_HIP;
-  // Launch shape: waves per tensor of the projections, timed once per (count, largest mode
-  // size): four fill the GPU best with many tensors, eight shorten each of a few.
-  const std::pair<int, int> key(count, nmax);
-  auto tuned = h->batch_tune.find(key);
-  if (tuned == h->batch_tune.end()) {
-    float best = 1e30f;
-    int pick = 4;
-    for (int waves : {4, 8}) {
-      if (hipEventRecord(h->ev[0], h->stream) != hipSuccess) return HT_ERR_HIP;
-      if (batch_ht_launch(h->stream, r, waves)) return HT_ERR_HIP;
-      if (hipEventRecord(h->ev[1], h->stream) != hipSuccess || hipEventSynchronize(h->ev[1]) != hipSuccess)
-        return HT_ERR_HIP;
-      float ms = 0.f;
-      (void)hipEventElapsedTime(&ms, h->ev[0], h->ev[1]);
-      if (ms < best) {
-        best = ms;
-        pick = waves;
-      }
-    }
-    tuned = h->batch_tune.emplace(key, pick).first;
-  }
-  const int waves = tuned->second;
   // The launch runs from a graph captured for these exact arguments once they come a second
   // time in a row; arguments that change from call to call (a new output each time) are
   // launched as they are, since capturing costs more than the launches it saves.
-  std::vector<const void*> bkey = {x, itd, ord, out, errd, r.gram, r.basis, (const void*)(intptr_t)count,
-                                   (const void*)(intptr_t)waves};
+  std::vector<const void*> bkey = {x, itd, ord, out, errd, r.gram, r.basis, (const void*)(intptr_t)count};
   for (int c = 0; c < BT_CLASSES; ++c) bkey.push_back((const void*)(intptr_t)r.eig_count[c]);
   const bool again = h->bkey == bkey;
   if (!again) {
@@ -189,13 +164,13 @@ ht_status ht_decompose_batched(ht_handle_t h, const float* x, int32_t count, con
     h->bkey = bkey;
   } else if (!h->bexec) {
     if (hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal) != hipSuccess) return HT_ERR_HIP;
-    const int ls = batch_ht_launch(h->stream, r, waves);
+    const int ls = batch_ht_launch(h->stream, r);
     const hipError_t ce = hipStreamEndCapture(h->stream, &h->bgraph);
     if (ls || ce != hipSuccess) return HT_ERR_HIP;
     if (hipGraphInstantiate(&h->bexec, h->bgraph, nullptr, nullptr, 0) != hipSuccess) return HT_ERR_HIP;
   }
   if (hipEventRecord(h->ev[0], h->stream) != hipSuccess) return HT_ERR_HIP;
-  if (h->bexec ? hipGraphLaunch(h->bexec, h->stream) != hipSuccess : batch_ht_launch(h->stream, r, waves) != 0)
+  if (h->bexec ? hipGraphLaunch(h->bexec, h->stream) != hipSuccess : batch_ht_launch(h->stream, r) != 0)
     return HT_ERR_HIP;
   if (hipEventRecord(h->ev[1], h->stream) != hipSuccess) return HT_ERR_HIP;
   if (rel_err &&

@@ -358,7 +358,7 @@ struct BatchRun {
 };
 // doubles of BatchItem::u_scr's block for a tensor of these mode sizes
 inline long batch_basis_size(int n1, int n2, int n3) { return (long)BT_RMAX * (n1 + n2 + n3 + 3) + 8; }
-int batch_ht_launch(hipStream_t st, const BatchRun& r, int waves);
+int batch_ht_launch(hipStream_t st, const BatchRun& r);
 // Bump tensor from its factors (n_bumps x order x n) and amplitudes. With sumsq != null
 // also sumsq[0] = ||x||^2 of the FP32 values, part holding gen_bumps_planes(order, n)
 // doubles (order >= 2, n <= 1024, n_bumps <= 8, x 16-byte aligned; else an error).

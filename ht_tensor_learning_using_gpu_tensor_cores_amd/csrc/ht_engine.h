@@ -1,7 +1,6 @@
 // Internal host-side types of the HT engine.
 #pragma once
 #include <atomic>
-#include <map>
 #include <utility>
 #include <vector>
 
@@ -297,9 +296,7 @@ struct ht_handle_s {
   float* obuf = nullptr;   // device output staging for host outputs
   size_t obuf_bytes = 0;
   ht::Profiler prof;
-  // batched entry point: autotuned launch shape per (count, largest mode size) and the
-  // graph of the last launch with the arguments it was captured for
-  std::map<std::pair<int, int>, int> batch_tune;
+  // batched entry point: the graph of the last launch with the arguments it was captured for
   hipGraph_t bgraph = nullptr;
   hipGraphExec_t bexec = nullptr;
   std::vector<const void*> bkey;

@@ -541,9 +541,14 @@ __global__ __launch_bounds__(64 * NW, 3) void batch_proj_kernel(BatchRun r) {
 }
 
 constexpr int BG_WHOLE = 1024;  // tensors from which a wave takes a whole Gram
+// Tensors from which a projection has four waves, not eight: two work-groups of eight a CU hold
+// fewer. A fixed rule, since the waves decide the order of sums and with it the last bits.
+// Whole call, 16 to 64 rows, eight / four: 40 tensors 0.955 / 0.982 ms, 400 1.965 / 2.026, 1000
+// 3.36 / 3.37, 4096 11.30 / 11.13; 8 to 24 rows: 400 0.294 / 0.295, 600 0.322 / 0.315.
+constexpr int BP_FOUR = 512;
 
-int batch_ht_launch(hipStream_t st, const BatchRun& r, int waves) {
-  if (r.count < 1 || (waves != 4 && waves != 8)) return 8;
+int batch_ht_launch(hipStream_t st, const BatchRun& r) {
+  if (r.count < 1) return 8;
   // whole Grams once their waves outnumber the 1024 SIMDs threefold
   const int panels = r.count >= BG_WHOLE ? 1 : 4;
   hipLaunchKernelGGL(batch_gram_kernel, dim3(24 * panels * ((r.count + 7) / 8)), dim3(64), 0, st, r, panels);
@@ -562,7 +567,7 @@ int batch_ht_launch(hipStream_t st, const BatchRun& r, int waves) {
     }
     first += n;
   }
-  if (waves == 4) hipLaunchKernelGGL(batch_proj_kernel<4>, dim3(r.count), dim3(256), 0, st, r);
+  if (r.count >= BP_FOUR) hipLaunchKernelGGL(batch_proj_kernel<4>, dim3(r.count), dim3(256), 0, st, r);
   else hipLaunchKernelGGL(batch_proj_kernel<8>, dim3(r.count), dim3(512), 0, st, r);
   return hipGetLastError() == hipSuccess ? 0 : 5;
 }
