@@ -553,9 +553,15 @@ int batch_ht_launch(hipStream_t st, const BatchRun& r) {
   const int panels = r.count >= BG_WHOLE ? 1 : 4;
   hipLaunchKernelGGL(batch_gram_kernel, dim3(24 * panels * ((r.count + 7) / 8)), dim3(64), 0, st, r, panels);
   int first = 0;
-  if (3 * r.count <= 512) {
-    // every problem resident at once in the largest class's LDS (two on each of 256 CUs): one
-    // launch, 16 waves a problem (40 tensors: 0.72 ms; class after class 2.0)
+  // One launch for every class, 16 waves a problem in the largest class's LDS, or the classes one
+  // after another, each as long as its longest problem. Up to 512 problems (two on each of 256
+  // CUs) all are resident at once: 40 tensors of 16 to 64 rows 0.96 ms, class after class 1.83.
+  // With both long classes in the batch the one launch stays ahead until twice as many: 171
+  // tensors 1.00 against 1.90, 300 1.55 / 2.00, 400 1.97 / 2.06, 600 2.88 / 2.58; of 48 to 64 rows
+  // 200 2.03 / 2.25, 300 2.82 / 2.84, 400 3.58 / 3.46. Without them it does not: of 8 to 24 rows 170
+  // 0.25 / 0.27, 200 0.30 / 0.28, 300 0.41 / 0.29.
+  const bool both_long = r.eig_count[2] > 0 && r.eig_count[3] > 0;
+  if (3 * r.count <= (both_long ? 1024 : 512)) {
     hipLaunchKernelGGL((batch_eig_kernel<64, 1024>), dim3(3 * r.count), dim3(1024), 0, st, r, 0);
   } else for (int c = BT_CLASSES - 1; c >= 0; --c) {  // the longest first
     const int n = r.eig_count[c];

@@ -48,3 +48,27 @@ def test_same_in_every_handle(count):
                 if first is None:
                     first = got, err
                 assert np.array_equal(got, first[0]) and np.array_equal(err, first[1])
+
+
+# Eigen problems of every size class, one launch for all (341 tensors) and a launch for each (342);
+# without the two long classes the line is at 170. The classes differ in threads a problem, so in
+# the order of the convergence test's sums: a sweep more or less, 1e-14 of the values.
+@pytest.mark.parametrize("sizes,low,high", [((16, 30, 40, 64), 341, 342), ((5, 16, 24, 32), 170, 171)])
+def test_eigen_launches(sizes, low, high):
+    import torch
+    rng = np.random.default_rng(9)
+    shapes = np.array([[sizes[i], sizes[(i + 1) % 4], sizes[(i + 2) % 4]] for i in range(4)], dtype=np.int64)
+    core = np.full((4, 3), 4, np.int32)
+    offs = np.concatenate([[0], np.cumsum(shapes.prod(1))]).astype(np.int64)
+    xd = torch.from_numpy(rng.standard_normal(offs[-1]).astype(np.float32)).cuda()
+    got = []
+    for count in (low, high):
+        pick = np.arange(count) % 4
+        res, err, _ = ht.decompose_batched(ht.Batch(shapes[pick], xd, offs[:-1][pick]),
+                                           np.ascontiguousarray(ht.batch_ranks(core)[pick]))
+        for b in range(4, count):
+            assert err[b] == err[b % 4] and torch.equal(res[b].packed, res[b % 4].packed), b
+        got.append(([r.packed.cpu().numpy() for r in res[:4]], err[:4]))
+    for b in range(4):
+        np.testing.assert_allclose(got[1][0][b], got[0][0][b], rtol=2e-6, atol=2e-6)
+        assert abs(got[1][1][b] - got[0][1][b]) <= 1e-9
