@@ -43,17 +43,17 @@ __device__ __forceinline__ double rsq_nr(double x) {
 }
 
 // Jacobi rotation (c, s) that annihilates a_pq (Rutishauser's form: t = tan(phi) of the
-// smaller angle, c = 1/sqrt(1 + t^2), s = t c; c^2 + s^2 = 1 to rounding). An a_pq whose angle
-// or reciprocal would leave the FP64 range (exactly dependent columns leave entries down to
-// the subnormal numbers, and NaN came of them) counts as zero.
+// smaller angle, c = 1/sqrt(1 + t^2), s = t c; c^2 + s^2 = 1 to rounding). Without one where
+// the cotangent leaves the FP64 range or is NaN: a_pq = 0, or so small that its reciprocal
+// overflows (exactly dependent columns leave entries down to the subnormal numbers).
 __device__ __forceinline__ void jacobi_rotation(double app, double aqq, double apq, double& c, double& s) {
   c = 1.0;
   s = 0.0;
-  const double d = aqq - app;
-  if (fabs(apq) <= fmax(1e-290, 1e-150 * fabs(d))) return;
-  const double tau = d * rcp_nr(2.0 * apq);
+  const double tau = (aqq - app) * rcp_nr(2.0 * apq);
+  const double at = fabs(tau);
+  if (!(at < 1e150)) return;
   const double h = 1.0 + tau * tau;
-  double t = rcp_nr(fabs(tau) + h * rsq_nr(h));
+  double t = rcp_nr(at + h * rsq_nr(h));
   if (tau < 0.0) t = -t;
   c = rsq_nr(1.0 + t * t);
   s = t * c;
