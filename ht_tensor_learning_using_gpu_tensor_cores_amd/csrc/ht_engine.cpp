@@ -365,8 +365,9 @@ int Engine::gram2(const float* x, PMS v1, PMS v2, int prec, double* G1, double* 
 
 // Top-k eigenpairs (descending, canonical signs) of `batch` symmetric PSD n x n FP64
 // matrices G (stride n*n), written to U (stride n*k) and w (stride k).
-// n <= 64: solved directly (k_tri.h, Jacobi for k > 32). n <= 256: rounds of block subspace iteration (block b,
-// Householder re-orthonormalisation, Rayleigh-Ritz with a b x b Jacobi solve) until
+// n <= 64: solved directly (k_tri.h, Jacobi for k > 32). n <= 256: rounds of block subspace
+// iteration (block b, CholeskyQR2 with Householder as fallback, Rayleigh-Ritz with a b x b Jacobi
+// solve) until
 // every top-k Ritz residual is below tol * theta_1. Round 0 applies q0 normalised powers
 // to a Gaussian block; later rounds restart from the previous Ritz basis and apply a
 // Chebyshev filter (degree 8, 16, ...) that damps [0, smallest Ritz value]. A missed
@@ -945,7 +946,8 @@ int Engine::svd_subspace(const float* x, PMS v, int kU, int kW, double* U, doubl
   ++eig_calls;
   // Y = Q R, R = Q^T Y = Q^T A Qz; sigma^2 and the left vectors of R from R R^T (its
   // eigenvectors are orthonormal whatever sigma, where those of Y^T Y would have to be divided
-  // by it)
+  // by it). TSQR's R is FP64; here Q is rounded to FP32 before the product, which moves sigma by
+  // ~3e-8 / sqrt(rows) of itself, under the 6e-8 of the FP32 output.
   CK(orth(Y, rows, Q, 3));
   if (!by_tsqr) {
     CK(tall_gram_launch(st, Q, b, Y, b, rows, part, R));
@@ -1338,7 +1340,8 @@ int Engine::run_plain(const float* x) {
       CK(eig_to_sv(w, t));
       if (adaptive) CK(choose_rank(t, w, k, adapt_xsq, 1));
     } else if (cols <= 1024 && (p.lo[t] == 0 || p.hi[t] == p.order)) {
-      // Gram of the complementary (contiguous) mode range, then U = X_(t) V / sigma via TSQR.
+      // Gram of the complementary (contiguous) mode range, then U spans X_(t) V by CholeskyQR
+      // (TSQR where a pivot fails).
       const PMS vc = p.lo[t] == 0 ? PMS{rows, cols, 1} : PMS{1, cols, rows};
       double* G = alloc<double>((size_t)cols * cols);
       double* Vc = alloc<double>((size_t)cols * k);

@@ -14,12 +14,13 @@
 //                (U1 and U2 (x) U3 orthonormal), all terms in FP64.
 // n <= 64, ranks <= 8.
 //
-// Kernels on one stream (one graph launch): Grams, eigen problems, projections. What bounds
+// Kernels on one stream: Grams, eigen problems, projections (from a hipGraph once the same
+// arguments come a second time in a row). What bounds
 // them differs: the Grams FP32 MFMA, the eigen problems barriers and instruction issue of
 // cyclic Jacobi, the projections FP64 MFMA. One persistent kernel that ran each tensor's
 // phases in turn held every phase to the occupancy of its largest and solved a tensor's three
-// eigen problems one after another: 4096 tensors of 16-64 rows 30.2 -> 12.0 ms (Grams 1.0,
-// eigen problems 10.6, projections 0.7), 40 of them 6.4 -> 0.88 ms.
+// eigen problems one after another: 4096 tensors of 16-64 rows 30.2 -> 11.1 ms (11.9 under the
+// profiler: Grams 1.0, eigen problems 10.4, projections 0.5), 40 of them 6.4 -> 0.95 ms.
 #include <algorithm>
 
 #include "k_tri.h"
@@ -325,10 +326,10 @@ __device__ __forceinline__ void eig_values(const EigTask& e, int j, double lam) 
 // descending size: cyclic Jacobi, then the top k columns with canonical signs. The class sets
 // the LDS, and with it the problems per CU that hide each other's barriers and chains: 67 KB
 // for 64 rows, 38 KB for 48, 17 KB for 32, 5 KB for 16.
-// (The one-wave tridiagonal solver of the single decompositions takes 1.7 ms here, but it
-// moves the relative error, an FP64 result that cancels to 1e-6 of ||X||^2: Jacobi's rotations
-// leave the bases' squared norms at 1 + 1e-14, and the error 2e-8 of itself away from what an
-// exactly orthonormal basis gives.)
+// (The one-wave tridiagonal solver of the single decompositions takes 1.7 ms here, but with it
+// the reported relative error moves by 2e-8 of itself: the formula above takes the bases as
+// exactly orthonormal and cancels to 1e-6 of ||X||^2, so their squared norms' 1 + 1e-14 shows. A
+// quadratic term with the bases' own Grams would cancel that and let the faster solver in.)
 // Measured per class at 4096 tensors: 64 rows 8.7 ms with 256 threads a problem, 7.2 with 512;
 // 48 rows 2.5 and 2.66.
 template <int NC, int NT>

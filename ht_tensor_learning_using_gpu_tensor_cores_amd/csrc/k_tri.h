@@ -20,7 +20,8 @@
 // The result is checked before it is used: residuals in the tridiagonal basis, and mutual
 // orthogonality of the k vectors, which twisted vectors of clustered eigenvalues (ranks
 // above the numerical rank) lack and a Gram-Schmidt pass restores. Exactly equal
-// eigenvalues fail the check and the caller takes Jacobi.
+// eigenvalues fail the check and the caller takes Jacobi (rounding usually separates them:
+// 64^4 with rotated identity factors stays in this solver's time).
 #pragma once
 #include "k_jacobi.h"
 
@@ -251,7 +252,9 @@ __device__ __forceinline__ void tri_sections(int n, int k, TriLds* __restrict__ 
       const double x0 = fma(step, (double)(jg + 1), lo), x1 = fma(step, (double)(jg + 1 + G), lo);
       // p_i = (d_i - x) p_{i-1} - e_{i-1}^2 p_{i-2}: its sign changes count the eigenvalues
       // below x. The pair is rescaled by a power of two every sixteen steps, over which it
-      // grows by at most 8^16 and shrinks by no more than the floor 1e-34 of e^2 every two.
+      // grows by less than (2 nrm + 1)^16 < 1e102 (d, x and e are within the norm's bound, which
+      // tri_reduce_wave holds under 1e6) and shrinks by no more than the floor 1e-34 of e^2
+      // every two.
       double am = 0.0, ac = 1.0, bm = 0.0, bc = 1.0;
       int nega = 0, negb = 0;
       unsigned sa = 0, sb = 0;  // signs, newest lowest

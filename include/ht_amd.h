@@ -267,9 +267,9 @@ ht_status ht_generate_bumps(ht_handle_t handle, int32_t order, int64_t n, int32_
                             uint64_t seed, int64_t sample, float* x_dev);
 
 /* ---- batched HT ------------------------------------------------------------------
- * Many small, unevenly sized 3rd-order tensors decomposed in one graph launch (Grams, eigen
- * problems, projections of all tensors; captured in a hipGraph and replayed while the
- * arguments stay the same), with the
+ * Many small, unevenly sized 3rd-order tensors decomposed by a few launches (Grams, eigen
+ * problems, projections of all tensors; the second call in a row with the same arguments
+ * captures them in a hipGraph, replayed while those stay the same), with the
  * tree {1},{2,3} (heap nodes: 0 = {1,2,3}, 1 = {1}, 2 = {2,3}, 3 = {2}, 4 = {3}) and
  * the plain semantics. No counterpart in the reference: its third_order_tensor_decompsition/
  * CUDA/Optimized/htd_batch.cu is a single decomposition and batch_tensorcore.cu:46-95 a
@@ -279,8 +279,9 @@ ht_status ht_generate_bumps(ht_handle_t handle, int32_t order, int64_t n, int32_
  *   out        device; tensor b's block, in ht_output_layout's order for that tree, at
  *              out + out_offsets[b] (ht_batch_output_layout gives a packed choice)
  *   rel_err    host, count relative errors (may be NULL)
- * The launch shape (waves per tensor of the projections) is timed once per (count,
- * largest mode size) on the first call and cached in the handle. */
+ * The launch shapes follow from the number of tensors and their sizes alone: the same call
+ * gives the same bits in every handle and process. Scratch memory grows with the batch, by up
+ * to 62 KB a tensor (its three leaf Grams in FP32, its leaf bases in FP64). */
 ht_status ht_batch_output_layout(int32_t count, const int64_t* dims, const int32_t* ranks,
                                  int64_t* out_offsets, int64_t* total);
 ht_status ht_decompose_batched(ht_handle_t handle, const float* x, int32_t count, const int64_t* dims,
